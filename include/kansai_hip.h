@@ -198,7 +198,9 @@ int kh_dequantize_packed(const int8_t* q_packed, int64_t k, int64_t n, const dou
  * accumulator exact.  Skinny shapes (M <= 64) whose 16-column tiles leave
  * CUs idle (N < 16 x CUs / 2) with K >= 8192 split K across workgroups:
  * int32 partials in pooled device memory, summed (exactly) by a second
- * launch that applies the epilogue. */
+ * launch that applies the epilogue; so do other products of few tiles with
+ * K >= 6144.  Large operands whose rows are no multiple of 64 bytes, or not
+ * 16-byte aligned, are first copied to such rows in pooled memory. */
 int kh_gemm_i8(const int8_t* a, const int8_t* b_packed, int64_t M, int64_t N, int64_t K,
                const double* sa, int sa_per_row, const double* sb, int sb_per_col,
                const float* bias, float* out, int32_t* acc_out);

@@ -12,14 +12,14 @@
 // Layout: a [M, K] row-major (activations, K-contiguous); b [N, K] row-major
 // (the packed weight, K-contiguous); out/acc [M, N] row-major.
 //
-// Structure: a workgroup owns a BM x BN output tile and walks K in BK steps.
-// Each step's A and B tiles are staged in LDS (double-buffered; the next
-// tile's global loads are in flight while the current one is multiplied).
-// Waves are arranged WM x WN; each wave owns (BM/WM) x (BN/WN) outputs as
-// 32x32 blocks of v_mfma_i32_32x32x32_i8 (one MFMA consumes 32 k: lane l
-// supplies 16 consecutive k of A row l%32 and of B column l%32).  LDS rows
-// are padded by 16 bytes so the 16-byte ds_read of 8 consecutive rows hits
-// distinct banks.
+// Kernels, by shape (gemm_i8_impl holds the rule):
+//   gemm_i8_pingpong_kernel   products that fill the chip with large tiles
+//   gemm_i8_tile_kernel       the others, and rows that are not 16-byte aligned
+//                             (kh_gemm_i8_tile.h)
+//   gemm_i8_skinny_kernel     few rows: the weight stream
+//   gemm_i8_narrow_kernel     many rows, few columns
+//   gemm_i8_small_kernel      operands of less than 16 bytes, and K = 0
+// All multiply on v_mfma_i32_*_i8 and share the epilogue below.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -311,143 +311,16 @@ __device__ __forceinline__ unsigned store_block32_full(const Epilogue& ep, int64
     return mx;
 }
 
-template <int BM, int BN, int BK, int WM, int WN>
-struct GemmCfg {
-    static constexpr int kThreads = WM * WN * 64;
-    static constexpr int kPad = 16;
-    static constexpr int kLdsRow = BK + kPad;  // bytes per LDS row
-    static constexpr int kWaveM = BM / WM;
-    static constexpr int kWaveN = BN / WN;
-    static constexpr int kTM = kWaveM / 32;
-    static constexpr int kTN = kWaveN / 32;
-    static constexpr int kChunksPerRow = BK / 16;
-    static constexpr int kAChunks = BM * kChunksPerRow / kThreads;  // 16-byte chunks per thread
-    static constexpr int kBChunks = BN * kChunksPerRow / kThreads;
-    static constexpr int kLdsA = BM * kLdsRow;
-    static constexpr int kLdsB = BN * kLdsRow;
-    static_assert(BM % (WM * 32) == 0 && BN % (WN * 32) == 0, "wave tile must be a multiple of 32");
-    static_assert(BK % 32 == 0, "BK must be a multiple of 32");
-    static_assert((BM * kChunksPerRow) % kThreads == 0 && (BN * kChunksPerRow) % kThreads == 0, "chunking");
-};
-
-// Loads one 16-byte chunk of a K-contiguous operand (zero outside the matrix).
-// VEC16: K % 16 == 0 and the base is 16-byte aligned, so a chunk is either
-// fully inside or fully outside; otherwise bytes are gathered one by one.
-template <bool VEC16>
-__device__ __forceinline__ i32x4 load_chunk(const int8_t* __restrict__ base, int64_t row, int64_t rows, int64_t k,
-                                            int64_t K) {
-    if (VEC16) {
-        if (row < rows && k < K) return *reinterpret_cast<const i32x4*>(base + row * K + k);
-        return i32x4{0, 0, 0, 0};
-    } else {
-        unsigned w[4] = {0, 0, 0, 0};
-        if (row < rows) {
-            const int8_t* p = base + row * K;
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                if (k + e < K) w[e >> 2] |= ((unsigned)(uint8_t)p[k + e]) << (8 * (e & 3));
-        }
-        return i32x4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-    }
-}
-
-template <int BM, int BN, int BK, int WM, int WN, bool VEC16>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_i8_kernel(const int8_t* __restrict__ A,
-                                                               const int8_t* __restrict__ B, int64_t M, int64_t N,
-                                                               int64_t K, Epilogue ep) {
-    using C = GemmCfg<BM, BN, BK, WM, WN>;
-    __shared__ __attribute__((aligned(16))) int8_t lds[2][C::kLdsA + C::kLdsB];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int wm = wave / WN;
-    const int wn = wave % WN;
-    const int64_t m0 = (int64_t)blockIdx.y * BM;
-    const int64_t n0 = (int64_t)blockIdx.x * BN;
-
-    i32x16 acc[C::kTM][C::kTN];
-#pragma unroll
-    for (int a = 0; a < C::kTM; ++a)
-#pragma unroll
-        for (int b = 0; b < C::kTN; ++b) acc[a][b] = i32x16{0};
-
-    i32x4 ra[C::kAChunks], rb[C::kBChunks];
-    auto gload = [&](int64_t k0) {
-#pragma unroll
-        for (int c = 0; c < C::kAChunks; ++c) {
-            const int idx = tid + c * C::kThreads;
-            const int r = idx / C::kChunksPerRow, kc = idx % C::kChunksPerRow;
-            ra[c] = load_chunk<VEC16>(A, m0 + r, M, k0 + kc * 16, K);
-        }
-#pragma unroll
-        for (int c = 0; c < C::kBChunks; ++c) {
-            const int idx = tid + c * C::kThreads;
-            const int r = idx / C::kChunksPerRow, kc = idx % C::kChunksPerRow;
-            rb[c] = load_chunk<VEC16>(B, n0 + r, N, k0 + kc * 16, K);
-        }
-    };
-    auto lstore = [&](int buf) {
-        int8_t* la = lds[buf];
-        int8_t* lb = lds[buf] + C::kLdsA;
-#pragma unroll
-        for (int c = 0; c < C::kAChunks; ++c) {
-            const int idx = tid + c * C::kThreads;
-            const int r = idx / C::kChunksPerRow, kc = idx % C::kChunksPerRow;
-            *reinterpret_cast<i32x4*>(la + r * C::kLdsRow + kc * 16) = ra[c];
-        }
-#pragma unroll
-        for (int c = 0; c < C::kBChunks; ++c) {
-            const int idx = tid + c * C::kThreads;
-            const int r = idx / C::kChunksPerRow, kc = idx % C::kChunksPerRow;
-            *reinterpret_cast<i32x4*>(lb + r * C::kLdsRow + kc * 16) = rb[c];
-        }
-    };
-
-    const int64_t nk = (K + BK - 1) / BK;
-    gload(0);
-    lstore(0);
-    __syncthreads();
-
-    const int frag_row = lane & 31;
-    const int frag_k = (lane >> 5) * 16;
-    for (int64_t kt = 0; kt < nk; ++kt) {
-        const int buf = (int)(kt & 1);
-        if (kt + 1 < nk) gload((kt + 1) * BK);
-        const int8_t* la = lds[buf] + (wm * C::kWaveM + frag_row) * C::kLdsRow + frag_k;
-        const int8_t* lb = lds[buf] + C::kLdsA + (wn * C::kWaveN + frag_row) * C::kLdsRow + frag_k;
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 32) {
-            i32x4 fa[C::kTM], fb[C::kTN];
-#pragma unroll
-            for (int a = 0; a < C::kTM; ++a) fa[a] = *reinterpret_cast<const i32x4*>(la + a * 32 * C::kLdsRow + kk);
-#pragma unroll
-            for (int b = 0; b < C::kTN; ++b) fb[b] = *reinterpret_cast<const i32x4*>(lb + b * 32 * C::kLdsRow + kk);
-#pragma unroll
-            for (int a = 0; a < C::kTM; ++a)
-#pragma unroll
-                for (int b = 0; b < C::kTN; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[a], fb[b], acc[a][b], 0, 0, 0);
-        }
-        if (kt + 1 < nk) lstore(buf ^ 1);
-        __syncthreads();
-    }
-
-    // 32x32 MFMA result layout: register r of lane l holds row
-    // 8*(r/4) + 4*(l/32) + r%4 and column l%32 of the block.
-    const int64_t row_base = m0 + wm * C::kWaveM + 4 * (lane >> 5);
-    const int64_t col_base = n0 + wn * C::kWaveN + (lane & 31);
-#pragma unroll
-    for (int a = 0; a < C::kTM; ++a)
-#pragma unroll
-        for (int b = 0; b < C::kTN; ++b) {
-            const int64_t j = col_base + b * 32;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int64_t i = row_base + a * 32 + 8 * (r >> 2) + (r & 3);
-                if (i < M && j < N) epilogue_store(ep, i, j, N, acc[a][b][r]);
-            }
-        }
+// Any product, one thread per output: operands of less than 16 bytes (the
+// other kernels load 16 at a time) and K = 0.
+__global__ __launch_bounds__(256) void gemm_i8_small_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
+                                                            int64_t M, int64_t N, int64_t K, Epilogue ep) {
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= M * N) return;
+    const int64_t i = idx / N, j = idx % N;
+    int32_t acc = 0;
+    for (int64_t k = 0; k < K; ++k) acc += (int32_t)A[i * K + k] * (int32_t)B[j * K + k];
+    epilogue_store(ep, i, j, N, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1406,6 +1279,20 @@ bool skinny_fits(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t
            kh::aligned(B, 16) && M * K <= 0xFFFFFFFFLL && N * K <= 0xFFFFFFFFLL && N <= 0x7FFFFFFF;
 }
 
+// Where the skinny kernel is faster than the 64 x 64 tiles
+// (kh_gemm_i8_tile.h): up to 16 rows everywhere; 17 to 32 except where a wide
+// weight takes several workgroups per CU, each reading its own copy of the
+// activations (M = 17, K = 8192, N = 11008: 26.2 against 20.3 us; K = 4096:
+// 13.4, 12.5; N = 4096: 7.5, 10.1); beyond, where four row tiles a wave halve
+// the workgroups in flight, only for short K and no more than one workgroup per
+// CU (M = 64, N = 4096: K = 512 4.0 against 4.4, 1536 6.4, 6.2, 4096 12.2, 9.7;
+// N = 11008: K = 512 6.9, 5.2, K = 1536 13.4, 6.9).
+bool skinny_pays(const kh::Device* d, int64_t M, int64_t N, int64_t K) {
+    if (M <= 16) return true;
+    const bool one_round = (N + 15) / 16 <= d->cus;
+    return M <= 32 ? one_round || K < 4096 : one_round && K < 1536;
+}
+
 // Split-K factor for a skinny launch: with one 16-column tile per workgroup a
 // narrow N leaves CUs idle (N = 1024: 64 workgroups on 256 CUs, each
 // streaming 16 K bytes of weight), so K is split over up to 8 workgroups per
@@ -1736,16 +1623,9 @@ bool pingpong_fits(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64
            ((M + 127) / 128) * ((N + 127) / 128) <= 0x7FFFFFFF;
 }
 
-template <int BM, int BN, int BK, int WM, int WN>
-int launch_gemm(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K, const Epilogue& ep,
-                bool vec16) {
-    dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((M + BM - 1) / BM));
-    if (vec16)
-        gemm_i8_kernel<BM, BN, BK, WM, WN, true><<<grid, WM * WN * 64, 0, d->stream>>>(A, B, M, N, K, ep);
-    else
-        gemm_i8_kernel<BM, BN, BK, WM, WN, false><<<grid, WM * WN * 64, 0, d->stream>>>(A, B, M, N, K, ep);
-    return kh::launch_status("gemm_i8");
-}
+}  // namespace
+#include "kh_gemm_i8_tile.h"
+namespace {
 
 // ---------------------------------------------------------------------------
 // Decode Linear for one to three tokens (kh_linear_i8 with M <= 3): the
@@ -2198,22 +2078,22 @@ static int gemm_i8_impl(const int8_t* a, const int8_t* b_packed, int64_t M, int6
     Epilogue ep{sa, sb, bias, out, acc_out, sa_per_row, sb_per_col, act, residual};
     int rc;
     bool parts_done = false;
-    if (skinny_fits(a, b_packed, M, N, K)) {
+    if (skinny_fits(a, b_packed, M, N, K) && skinny_pays(d, M, N, K)) {
         rc = launch_skinny(d, a, b_packed, M, N, K, ep, may_alloc);
     } else if (!parts && narrow_fits(a, b_packed, M, N, K)) {
         rc = launch_narrow(d, a, b_packed, M, N, K, ep);
-    } else if (pingpong_fits(a, b_packed, M, N, K)) {
+    } else if (M * K < 16 || N * K < 16) {
+        KH_REQUIRE(M * N <= 0x7FFFFFFFLL * 256, "kh_gemm_i8: shape too large");
+        gemm_i8_small_kernel<<<(unsigned)((M * N + 255) / 256), 256, 0, d->stream>>>(a, b_packed, M, N, K, ep);
+        rc = kh::launch_status("gemm_i8_small");
+    } else if (tile_pays(d, M, N, K) || !pingpong_fits(a, b_packed, M, N, K)) {
+        rc = launch_tile(d, a, b_packed, M, N, K, ep, may_alloc, parts, max_parts, nparts, &parts_done);
+    } else {
         // The ping-pong kernel writes one partial per workgroup when they fit.
         const int64_t worst = ((M + 127) / 128) * ((N + 127) / 128);
         const bool fused = parts && worst <= max_parts;
         rc = launch_pingpong(d, a, b_packed, M, N, K, ep, fused ? parts : nullptr, fused ? nparts : nullptr);
         parts_done = fused;
-    } else {
-        const bool vec16 = (K % 16 == 0) && kh::aligned(a, 16) && kh::aligned(b_packed, 16);
-        if (M >= 2048 && N >= 2048)
-            rc = launch_gemm<256, 256, 64, 2, 4>(d, a, b_packed, M, N, K, ep, vec16);
-        else
-            rc = launch_gemm<128, 128, 64, 2, 2>(d, a, b_packed, M, N, K, ep, vec16);
     }
     if (rc || !parts || parts_done) return rc;
     return kh_absmax_parts(out, M * N, parts, max_parts, nparts);

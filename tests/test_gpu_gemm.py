@@ -76,6 +76,51 @@ def test_gemm_i8_vs_oracle(hip, M, N, K):
     np.testing.assert_array_equal(bits32(out[rows]), bits32(eout))
 
 
+TILE_SHAPES = [
+    (63, 65, 127), (64, 64, 128), (65, 63, 129), (128, 130, 255), (70, 300, 5), (17, 16, 1), (33, 1, 40),  # edges
+    (16, 1, 1), (3, 5, 2), (1, 15, 1),                                  # operands of less than 16 bytes
+    (65, 70, 16), (300, 900, 112), (129, 64, 1040), (66, 200, 656),     # K % 16 == 0: a last stage partly past K
+    (40, 64, 6144), (100, 33, 11008), (65, 130, 6160), (70, 65, 6151),  # split over 4, 8, 4 and 4 workgroups
+    (8, 300, 11008), (3, 4096, 704),                                    # few rows, K no multiple of 512
+    (1700, 1700, 208), (1300, 2000, 384),                               # 128 x 64 tiles
+    (2100, 2100, 65), (2600, 2600, 80), (2600, 2600, 77),               # rows padded first: tiles, ping-pong
+]
+
+
+@pytest.mark.parametrize("M,N,K", TILE_SHAPES)
+def test_gemm_i8_tiles(hip, M, N, K):
+    """The products the ping-pong kernel's tiles do not fit, bit-exact (integer
+    sums): fp32 output alone, int32 alone, and the fused residual with its absmax
+    partials; operands at an odd address give the same bits."""
+    H, D = hip
+    gen = np.random.Generator(np.random.PCG64(M * 7919 + N * 31 + K))
+    a = gen.integers(-127, 128, (M, K), dtype=np.int8)
+    bt = gen.integers(-127, 128, (N, K), dtype=np.int8)
+    sa, sb = gen.uniform(1e-3, 5e-2, M), gen.uniform(1e-3, 5e-2, N)
+    bias = gen.standard_normal(N).astype(np.float32)
+    residual = gen.standard_normal((M, N)).astype(np.float32)
+    rows = np.arange(M) if M * N * K <= 2 ** 28 else np.sort(gen.choice(M, size=64, replace=False))
+    eacc = O.ko_gemm_i8(a[rows], bt)
+    eout = O.ko_epilogue(eacc, sa[rows], sb, bias)
+    dsa, dsb, dbias = D.from_host(sa), D.from_host(sb), D.from_host(bias)
+
+    def operand(x, shift):
+        flat = D.from_host(np.concatenate([np.full(shift, 99, np.int8), x.reshape(-1)]))
+        return flat.view(shift, x.shape)
+
+    for shift in (0, 3):
+        da, db = operand(a, shift), operand(bt, shift)
+        out, _ = H.gemm_i8(da, db, dsa, dsb, dbias)
+        np.testing.assert_array_equal(bits32(out.numpy()[rows]), bits32(eout))
+    _, acc = H.gemm_i8(operand(a, 0), operand(bt, 0), want_out=False, want_acc=True)
+    np.testing.assert_array_equal(acc.numpy()[rows], eacc)
+    out, parts = H.gemm_i8_fused(operand(a, 0), operand(bt, 0), dsa, dsb, dbias, residual=D.from_host(residual),
+                                 absmax=True)
+    got = out.numpy()
+    np.testing.assert_array_equal(bits32(got[rows]), bits32(residual[rows] + eout))
+    assert parts.buf.numpy()[:parts.count].max() == bits32(np.abs(got)).max()
+
+
 def test_gemm_i8_per_tensor_scales_and_no_bias(hip):
     H, D = hip
     gen = np.random.Generator(np.random.PCG64(12))
