@@ -335,6 +335,15 @@ int kh_dequantize_acc(const int32_t* acc, int64_t M, int64_t N, const double* sa
 int kh_matmul_f32(const float* a, const float* b, float* out, int64_t M, int64_t K, int64_t N,
                   const float* bias);
 
+/* The reference's weight-only Linear (quantize.py:115-122):
+ * out[i, j] = sum_k x[i, k] * dequantize(q_packed)[k, j] + bias[j], x fp32
+ * [M, K], q_packed int8 [N, K] with 1 or N binary64 scales, without the fp32
+ * weight being written.  Agrees with kh_dequantize_packed + kh_matmul_f32 to
+ * their rounding bound (the weights here are exact, the scale multiplies the
+ * sum); pooled device memory holds x as three bf16 parts. */
+int kh_linear_w8(const float* x, int64_t M, int64_t K, const int8_t* q_packed, int64_t N, const double* scales,
+                 int64_t scales_n, const float* bias, float* out);
+
 /* ---- fp32 elementwise around the path ----------------------------------- */
 
 /* out[i] = a[i] + b[i]: kan::metal::add (MetalOps.hpp:51),

@@ -24,34 +24,12 @@
 //   int32 sums as partial y (skinny_splitk_epilogue_kernel adds them up).
 #pragma once
 
+#include "kh_rows.h"
+
 namespace {
 
-typedef i32x4 i32x4_any __attribute__((aligned(1)));
-
-// The 16 bytes v of an operand chunk, of which the first `sh` belong to the
-// bytes before it (the load was pulled back by sh) and only `n` are wanted.
-__device__ __forceinline__ i32x4 tail_bytes(i32x4 v, int sh, int n) {
-    typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
-    u64x2 w = __builtin_bit_cast(u64x2, v);
-    unsigned long long lo = w.x, hi = w.y;
-    if (sh >= 8) {
-        lo = hi;
-        hi = 0;
-        sh -= 8;
-    }
-    if (sh >= 8) lo = 0;
-    else if (sh > 0) {
-        lo = (lo >> (8 * sh)) | (hi << (64 - 8 * sh));
-        hi >>= 8 * sh;
-    }
-    if (n <= 0) lo = 0;
-    else if (n < 8) lo &= (1ull << (8 * n)) - 1;
-    if (n <= 8) hi = 0;
-    else if (n < 16) hi &= (1ull << (8 * (n - 8))) - 1;
-    w.x = lo;
-    w.y = hi;
-    return __builtin_bit_cast(i32x4, w);
-}
+using kh::rows::i32x4_any;
+using kh::rows::tail_bytes;
 
 template <int BM, int BN, int NS, bool FUSED, bool DMA>
 __global__ __launch_bounds__(256, (BM + BN) * 128 * NS <= 53248 ? 3 : (BM + BN) * 128 * NS <= 81920 ? 2 : 1) void gemm_i8_tile_kernel(
@@ -365,23 +343,6 @@ bool tile_pays(const kh::Device* d, int64_t M, int64_t N, int64_t K) {
     return tiles64(M, N) <= 6 * (int64_t)d->cus && K <= 0x7FFFFFFF / 128 && M <= 0x7FFFFFFF && N <= 0x7FFFFFFF;
 }
 
-// Both operands' rows copied to a stride of Kp bytes (a multiple of 16, zeros
-// past K), 16 bytes a thread: row r of A, then of B.
-__global__ __launch_bounds__(256) void pad_rows_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
-                                                       int M, int N, int K, int Kp, int8_t* __restrict__ out) {
-    const int chunks = Kp / 16;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t row = idx / chunks;
-    if (row >= (int64_t)M + N) return;
-    const int k = (int)(idx - row * chunks) * 16;
-    const int8_t* const base = row < M ? A : B;
-    const int64_t off = (row < M ? row : row - M) * K + k, last = (int64_t)(row < M ? M : N) * K - 16;
-    const int64_t at = min(off, last);
-    i32x4 v = *reinterpret_cast<const i32x4_any*>(base + at);
-    if (k + 16 > K) v = tail_bytes(v, (int)(off - at), K - k);
-    *reinterpret_cast<i32x4*>(out + idx * 16) = v;
-}
-
 int launch_pingpong(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
                     const Epilogue& ep_in, unsigned* parts, int* nparts, int mode);
 
@@ -418,8 +379,8 @@ int launch_tile(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, int6
         if (rc) return rc;
         int8_t* const pa = static_cast<int8_t*>(pad);
         int8_t* const pb = pa + M * Kp;
-        pad_rows_kernel<<<(unsigned)(((M + N) * (Kp / 16) + 255) / 256), 256, 0, d->stream>>>(A, B, (int)M, (int)N,
-                                                                                              (int)K, (int)Kp, pa);
+        kh::rows::pad_rows_kernel<<<(unsigned)(((M + N) * (Kp / 16) + 255) / 256), 256, 0, d->stream>>>(
+            A, B, (int)M, (int)N, (int)K, (int)Kp, pa);
         rc = kh::launch_status("pad_rows");
         if (!rc) {
             const bool fused = parts && ((M + 127) / 128) * ((N + 127) / 128) <= max_parts;

@@ -263,6 +263,27 @@ def matmul(a: DeviceTensor, b: DeviceTensor, bias: DeviceTensor | None = None) -
     return out
 
 
+def linear_w8(x: DeviceTensor, b_packed: DeviceTensor, sb: DeviceTensor,
+              bias: DeviceTensor | None = None) -> DeviceTensor:
+    """matmul(x, dequantize_packed(b_packed, sb), bias) without the fp32
+    weight: x [..., K] fp32, b_packed [N, K] int8, out [..., N]."""
+    M, K, lead = _rows(x, "float32", "matmul(a)")
+    _need(b_packed, "int8", 2, "linear_w8(w)")
+    _need(sb, "float64", 1, "dequantize_packed(scales)")
+    Nn, K2 = b_packed.shape
+    if sb.shape[0] not in (1, Nn):
+        raise RuntimeError("dequantize_packed: scales must have 1 or out entries")
+    if K != K2:
+        raise RuntimeError("matmul: incompatible shapes")
+    if bias is not None:
+        _need(bias, "float32", 1, "matmul(bias)")
+        if bias.shape[0] != Nn:
+            raise RuntimeError("matmul: bias must have N entries")
+    out = DeviceTensor(lead + [Nn], "float32")
+    N.call("kh_linear_w8", x.ptr, M, K, b_packed.ptr, Nn, sb.ptr, sb.shape[0], _opt(bias), out.ptr)
+    return out
+
+
 def add(a: DeviceTensor, b: DeviceTensor) -> DeviceTensor:
     _need(a, "float32", None, "add")
     _need(b, "float32", None, "add")

@@ -541,6 +541,26 @@ def _dequantize(v):
     raise TypeError(f"dequantize: unsupported operand {type(v).__name__}")
 
 
+def _packed_weight_uses(graph, by_id) -> set:
+    """The dequantize nodes whose value only ever is a matmul's right operand:
+    where such a node's input is a packed weight, the matmul multiplies its
+    codes (kh_linear_w8) as the eager QLinear does, and the fp32 weight is not
+    written."""
+    nodes = {n.id for n in graph.nodes if n.op == "dequantize" and n.id != graph.output}
+    for n in graph.nodes:
+        for pos, i in enumerate(n.inputs):
+            if i in nodes and not (n.op in ("matmul", "matmul_bias") and pos == 1):
+                nodes.discard(i)
+    return nodes
+
+
+def _matmul(a, b, bias=None):
+    from .quantize import QTensor
+    if isinstance(b, QTensor):
+        return H.linear_w8(a, b.codes, b.scales, bias)
+    return H.matmul(a, b, bias)
+
+
 def _add(a, b):
     if list(a.shape) == list(b.shape):
         return H.add(a, b)
@@ -579,10 +599,9 @@ def _int8_operands(qa, qb, what):
 def _exec(node, vals):
     op = node.op
     ins = [vals[i] for i in node.inputs]
-    if op == "matmul":
-        return H.matmul(*ins)
-    if op == "matmul_bias":
-        return H.matmul(ins[0], ins[1], ins[2])
+    if op in ("matmul", "matmul_bias"):
+        # (a packed weight: _packed_weight_uses)
+        return _matmul(*ins)
     if op == "add":
         return _add(*ins)
     if op == "relu":
@@ -720,12 +739,14 @@ def _to_host(v):
 def _run(graph, args, plan, to_host, observe=None, capturing=False):
     if not N.available():
         raise RuntimeError("run_hip: no gfx950 (MI355X) device available on this system")
+    from .quantize import QTensor
     by_id = {n.id: n for n in graph.nodes}
     vals = {}
     for nid, a in zip(graph.inputs, args):
         dt = by_id[nid].dtype if by_id[nid].dtype in ("float32", "int32") else "float32"
         vals[nid] = a if isinstance(a, DeviceTensor) else DeviceTensor.from_host(as_host_array(a, dt))
     external = set(graph.inputs)
+    as_codes = _packed_weight_uses(graph, by_id)
     for idx, node in enumerate(graph.nodes):
         if node.op == "placeholder":
             continue
@@ -734,9 +755,15 @@ def _run(graph, args, plan, to_host, observe=None, capturing=False):
             if observe is not None:
                 observe(node, vals[node.id])
             continue
-        vals[node.id] = _exec(node, vals)
+        src = vals[node.inputs[0]] if node.id in as_codes else None
+        if isinstance(src, QTensor) and src.packed:
+            # Not its owner: the plan releases this value, never the weight.
+            vals[node.id] = QTensor(src.codes, src.scales, src.shape, src.granularity, packed=True, owned=False)
+        else:
+            vals[node.id] = _exec(node, vals)
         if observe is not None:
-            observe(node, vals[node.id])
+            seen = vals[node.id]
+            observe(node, seen.dequantize() if src is not None and isinstance(seen, QTensor) else seen)
         if plan is not None:
             for i in node.inputs:
                 src = by_id[i]

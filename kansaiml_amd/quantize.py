@@ -137,12 +137,14 @@ def dequantize(q, scale: float, shape) -> np.ndarray:
 
 def qlinear(x, qweight: QTensor, bias):
     """quantize.py:115-122: x.matmul(dequantize(W)).add(bias) -- the
-    reference's weight-only path -- with the dequantize and the fp32 GEMM (+
-    bias in its store) on the GPU.  Returns a DeviceTensor."""
+    reference's weight-only path -- on the GPU: a packed weight is multiplied
+    as its codes (kh_linear_w8), any other is dequantized for the fp32 GEMM (+
+    bias in its store).  Returns a DeviceTensor."""
     xd = to_device(x, "float32")
-    w = qweight.dequantize()
     b = to_device(bias, "float32") if bias is not None else None
-    return H.matmul(xd, w, b)
+    if qweight.packed:
+        return H.linear_w8(xd, qweight.codes, qweight.scales, b)
+    return H.matmul(xd, qweight.dequantize(), b)
 
 
 class QLinear:

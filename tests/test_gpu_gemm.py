@@ -87,6 +87,59 @@ TILE_SHAPES = [
 ]
 
 
+@pytest.mark.parametrize("M,N,K,col", [
+    (1, 16, 1, False), (3, 2, 5, True), (1, 100, 64, False), (5, 63, 65, True), (64, 64, 128, False),   # edges
+    (65, 129, 200, True), (33, 300, 1000, False), (7, 1000, 4096, True), (2, 70, 4101, False),          # K split
+    (1100, 1500, 96, True), (1030, 2050, 333, False), (11000, 24, 4100, True)])   # 64 x 128 tiles; two row slabs
+def test_linear_w8(hip, M, N, K, col):
+    """fp32 x (int8 weight): within the fp32 matmul's own bound of binary64,
+    with rows of any magnitude, zero rows, and rows of a range that the split
+    into bf16 parts cannot hold."""
+    H, D = hip
+    gen = np.random.Generator(np.random.PCG64(M * 7919 + N * 31 + K))
+    x = gen.standard_normal((M, K)).astype(np.float32)
+    q = gen.integers(-127, 128, (N, K), dtype=np.int8)
+    s = gen.uniform(1e-3, 5e-2, N if col else 1)
+    bias = gen.standard_normal(N).astype(np.float32)
+    with np.errstate(over="ignore", under="ignore"):
+        for i, f in enumerate((1.0, 1e30, 1e-30, 0.0, 1e-38)):
+            if i < M and M > 1:
+                x[i] *= np.float32(f)
+        if M > 5 and K > 2:  # 2^230 apart: a large value times a zero code beside tiny ones
+            x[5] *= np.float32(1e-35)
+            x[5, 0] = 3e34
+            q[::2, 0] = 0
+    out = H.linear_w8(D.from_host(x), D.from_host(q), D.from_host(s), D.from_host(bias)).numpy()
+    plain = H.matmul(D.from_host(x), H.dequantize_packed(D.from_host(q), D.from_host(s)), D.from_host(bias)).numpy()
+    rows = np.arange(M) if M * N * K <= 2 ** 27 else np.r_[:6, gen.choice(M, size=40, replace=False)]
+    w = q.T.astype(np.float64) * s
+    exact, size = x[rows].astype(np.float64) @ w, np.abs(x[rows]).astype(np.float64) @ np.abs(w)
+    # Binary32 sums of K exact products, the bias's rounding, and one step of the smallest binary32.
+    bound = 2 * K * 2.0 ** -24 * size + 2.0 ** -23 * np.abs(bias + exact) + 2.0 ** -149
+    err = np.abs(out[rows] - (exact + bias))
+    assert (err <= bound).all(), (err - bound).max()
+    assert np.linalg.norm(err) <= 1.5 * np.linalg.norm(plain[rows] - (exact + bias)) + np.linalg.norm(bound) * 0.01
+
+
+@pytest.mark.parametrize("M,N,K", [(4, 40, 64), (70, 300, 257)])
+def test_linear_w8_nonfinite(hip, M, N, K):
+    """Infinities and NaN where the fp32 product gives them."""
+    H, D = hip
+    gen = np.random.Generator(np.random.PCG64(K))
+    x = gen.standard_normal((M, K)).astype(np.float32)
+    q = gen.integers(-127, 128, (N, K), dtype=np.int8)
+    x[0, 3], x[1, K - 1], x[2, 0], x[2, 1] = np.inf, np.nan, np.inf, -np.inf
+    x[0, 4] = 3e38
+    q[::3, 3] = 0
+    s = np.array([0.02])
+    out = H.linear_w8(D.from_host(x), D.from_host(q), D.from_host(s)).numpy()
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ (q.T.astype(np.float64) * s)
+    np.testing.assert_array_equal(np.isnan(out), np.isnan(want))
+    np.testing.assert_array_equal(out[np.isinf(want)], want[np.isinf(want)])
+    assert np.isfinite(out[3:]).all()
+
+
 @pytest.mark.parametrize("M,N,K", TILE_SHAPES)
 def test_gemm_i8_tiles(hip, M, N, K):
     """The products the ping-pong kernel's tiles do not fit, bit-exact (integer
