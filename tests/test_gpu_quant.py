@@ -148,6 +148,28 @@ def test_quantize_weight_packed_vs_oracle(hip, k, n):
     assert s1.numpy()[0] == es1
 
 
+@pytest.mark.parametrize("k,n,shift", [
+    (1, 1, 0), (3, 5, 0), (127, 63, 0), (128, 64, 0), (129, 68, 0), (130, 68, 1), (16, 4, 0), (257, 260, 0),  # tile edges
+    (1001, 1000, 0), (5000, 12, 0), (700, 1001, 3), (20, 300000, 0), (300, 70000, 0)])  # 8 rows at a time; few partials
+def test_quantize_weight_packed_edges(hip, k, n, shift):
+    """Tile and unroll remainders of the packing kernels, zero columns and exact
+    ties; `shift` floats of misalignment take the scalar loads."""
+    H, D = hip
+    gen = np.random.Generator(np.random.PCG64(k * 31 + n))
+    w = (gen.standard_normal((k, n), dtype=np.float32) * np.float32(0.02))
+    w[:, n // 2] = 0.0
+    w[:, n // 3] = np.round(w[:, n // 3] * 1000) / np.float32(2)
+    wd = D.from_host(np.concatenate([np.full(shift, 9, np.float32), w.reshape(-1)])).view(shift, [k, n])
+    eq, es = O.ko_quantize_cols_packed(w)
+    q, s = H.quantize_cols_packed(wd)
+    np.testing.assert_array_equal(q.numpy(), eq)
+    np.testing.assert_array_equal(s.numpy(), es)
+    eq1, es1 = O.ko_quantize_tensor_packed(w)
+    q1, s1 = H.quantize_tensor_packed(wd)
+    np.testing.assert_array_equal(q1.numpy(), eq1)
+    assert s1.numpy()[0] == es1
+
+
 def test_misaligned_pointers_take_exact_generic_path(hip):
     """Offsets that break 16-byte alignment route to the scalar kernels."""
     H, D = hip
