@@ -370,13 +370,36 @@ __global__ __launch_bounds__(256, 1) void gemm_w8_kernel(const __bf16* __restric
         }
 }
 
-// The K splits' sums, in order, and the epilogue.
-__global__ __launch_bounds__(256) void w8_sum_kernel(int S, int64_t M, int64_t N, W8Out o) {
-    const int64_t mn = M * N, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// The K splits' sums, in order, and the epilogue.  Every split's load is issued
+// before the first is used; a thread takes V = 4 columns where N % 4 == 0.
+template <int S, int V>
+__global__ __launch_bounds__(256) void w8_sum_kernel(int M, int N, W8Out o) {
+    typedef float fv __attribute__((ext_vector_type(V == 4 ? 4 : 2)));
+    const int64_t mn = (int64_t)M * N, idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
     if (idx >= mn) return;
-    float sum = o.partial[idx];
-    for (int s = 1; s < S; ++s) sum += o.partial[s * mn + idx];
-    o.out[idx] = w8_value(o, sum, idx / N, idx % N);
+    fv p[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        if constexpr (V == 4) p[s] = *reinterpret_cast<const fv*>(o.partial + s * mn + idx);
+        else p[s].x = o.partial[s * mn + idx];
+    }
+    const int64_t i = idx / N, j = idx - i * N;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        float sum = p[0][u];
+#pragma unroll
+        for (int s = 1; s < S; ++s) sum += p[s][u];
+        o.out[idx + u] = w8_value(o, sum, i, j + u);
+    }
+}
+
+template <int S>
+int launch_w8_sum(kh::Device* d, int64_t M, int64_t N, const W8Out& o) {
+    if (N % 4 == 0)
+        w8_sum_kernel<S, 4><<<(unsigned)((M * N / 4 + 255) / 256), 256, 0, d->stream>>>((int)M, (int)N, o);
+    else
+        w8_sum_kernel<S, 1><<<(unsigned)((M * N + 255) / 256), 256, 0, d->stream>>>((int)M, (int)N, o);
+    return kh::launch_status("w8_sum");
 }
 
 template <int BM, int BN, int NS>
@@ -428,7 +451,7 @@ extern "C" int kh_linear_w8(const float* x, int64_t M, int64_t K, const int8_t* 
     while (!wide && S < 8 && tiles * S * 2 <= 2 * cus && steps >= 8 * S) S *= 2;
     const size_t planes_bytes = (size_t)(3 * slab * Kp) * sizeof(__bf16);
     const size_t factors_at = planes_bytes, codes_at = factors_at + (size_t)(slab + 1) / 2 * 2 * sizeof(double);
-    const size_t sums_at = codes_at + (pad ? (size_t)(N * Kp) : 0);
+    const size_t sums_at = codes_at + (pad ? (size_t)(N * Kp) : 0);  // (a multiple of 16)
     void* work = nullptr;
     int rc = kh_alloc(sums_at + (S > 1 ? (size_t)S * (size_t)(slab * N) * sizeof(float) : 0), &work);
     if (rc) return rc;
@@ -456,10 +479,9 @@ extern "C" int kh_linear_w8(const float* x, int64_t M, int64_t K, const int8_t* 
         const int64_t kq = pad ? Kp : K;
         rc = wide ? launch_w8<64, 128, 2>(d, planes, q, m, N, kq, Kp, S, o)
                   : launch_w8<64, 64, 2>(d, planes, q, m, N, kq, Kp, S, o);
-        if (!rc && S > 1) {
-            w8_sum_kernel<<<(unsigned)((m * N + 255) / 256), 256, 0, d->stream>>>(S, m, N, o);
-            rc = kh::launch_status("w8_sum");
-        }
+        if (!rc && S > 1)
+            rc = S == 2 ? launch_w8_sum<2>(d, m, N, o) : S == 4 ? launch_w8_sum<4>(d, m, N, o)
+                                                                : launch_w8_sum<8>(d, m, N, o);
     }
     kh_free(work);  // stream-ordered: reused only by work queued after the product
     return rc;
