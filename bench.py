@@ -49,9 +49,10 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-# MI355X published peaks (dense): int8 5.0 POP/s, fp32 157.3 TFLOP/s, HBM 8 TB/s.
+# MI355X published peaks (dense): int8 5.0 POP/s, bf16 2.5 PFLOP/s, HBM 8 TB/s.
+# A binary32 product is six bf16 ones (kh_gemm_f32x.h; the fp32 MFMA's peak is 157.3 TFLOP/s).
 PEAK_INT8_TOPS = 5000.0
-PEAK_FP32_TFLOPS = 157.3
+PEAK_FP32_TFLOPS = 2500.0 / 6
 PEAK_HBM_GBS = 8000.0
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 

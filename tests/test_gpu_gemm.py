@@ -593,6 +593,54 @@ def test_matmul_f32_vs_reference(hip, M, K, N):
         assert np.abs(got - ref).max() < 1e-3
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 4100), (2, 63, 33), (3, 128, 31), (7, 129, 1000), (16, 260, 512), (13, 4097, 700), (5, 64, 20000),
+    (17, 64, 64), (32, 300, 90),                                               # few rows
+    (33, 65, 63), (64, 130, 129), (65, 63, 1000), (40, 409, 4096),                # 64 x 64, K split
+    (1030, 1100, 70), (1000, 1000, 640), (2050, 2046, 200), (2600, 2570, 65), (3300, 3200, 130)])  # every tile
+def test_matmul_f32_tiles(hip, M, N, K):
+    """Every tile of the split product, within binary32's bound of binary64,
+    with all-tiny rows, values beyond the parts' range, infinities and NaN where
+    binary32 gives them, and operands at an odd address."""
+    H, D = hip
+    gen = np.random.Generator(np.random.PCG64(M * 7919 + N * 31 + K))
+    a, b = gen.standard_normal((M, K)).astype(np.float32), gen.standard_normal((K, N)).astype(np.float32)
+    bias = gen.standard_normal(N).astype(np.float32)
+
+    def put(x, shift=0):
+        return D.from_host(np.concatenate([np.full(shift, 9, np.float32), x.reshape(-1)])).view(shift, x.shape)
+
+    def check(a, b, bias, shift=0):
+        got = H.matmul(put(a, shift), put(b, shift), put(bias) if bias is not None else None).numpy()
+        with np.errstate(all="ignore"):
+            rows = np.arange(M) if M * N * K <= 2 ** 28 else np.r_[:40, gen.choice(M, size=40, replace=False)]
+            want = a[rows].astype(np.float64) @ b.astype(np.float64) + (0 if bias is None else bias)
+            size = np.abs(a[rows]).astype(np.float64) @ np.abs(b).astype(np.float64)
+            # Binary32 sums of K products (each rounded once), the bias's rounding, the smallest binary32.
+            bound = 2 * K * 2.0 ** -24 * size + 2.0 ** -23 * np.abs(want) + 2.0 ** -149
+            far = np.abs(got[rows] - want)
+            fin = np.isfinite(size) & (size < 1e38)
+            assert (far[fin] <= bound[fin]).all(), (far[fin] - bound[fin]).max()
+            bad = ~np.isfinite(want) & ~(size < 1e38)
+            np.testing.assert_array_equal(np.isnan(got[rows])[bad], np.isnan(want)[bad])
+            np.testing.assert_array_equal(got[rows][bad & ~np.isnan(want)], want[bad & ~np.isnan(want)])
+
+    check(a, b, bias)
+    check(a, b, None, shift=1)
+    check(a * np.float32(1e-20), b * np.float32(1e-15), None)  # every product below 2^-90
+    wild = a.copy()
+    wild[0] *= np.float32(1e30)
+    wild[M // 2] *= np.float32(1e-33)
+    wild[M - 1, K // 2] = 1e-36
+    wb = b.copy()
+    wb[K // 3, N // 2] = 2e18
+    check(wild, wb, bias)
+    if M > 2:
+        wild[1, K - 1], wild[2, 0], wild[M - 1, 0] = np.inf, np.nan, -np.inf
+        wb[K - 1, ::3] = 0.0
+        check(wild, wb, bias)
+
+
 def test_matmul_f32_c3b_full_size(hip):
     """Config C3b: M=N=K=4096 ~N(0,1); sampled rows against float64."""
     H, D = hip
