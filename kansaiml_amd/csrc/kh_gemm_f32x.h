@@ -7,8 +7,9 @@
 // products of two such triples six are multiplied, all exact: hh, hm, mh, hl, lh,
 // mm.  The other three are below 2^-24 of the product, less than the rounding of
 // one binary32 sum, and a product of sixteen k rounds six sums where the fp32
-// instruction rounds eight: the error against binary64 is smaller than the fp32
-// MFMA kernel's over every size measured (K = 64: 0.6 of it, 2048: 0.5).
+// instruction rounds eight: the error against binary64 is 0.83-0.92 of the fp32
+// MFMA kernel's at every size measured (K = 64 to 4096), 0.3-0.7 where K is split.
+// 4096^3: 1011 -> 792 us; 2000 x 4096 x 2048 298 -> 222; 190 x 72 x 512 52 -> 13.
 //
 // Two launches, and a sum of partials where K is split:
 //   split_units_kernel  A and B as planes [3, M, Kp] and [3, N, Kp] (B transposed:
@@ -434,7 +435,9 @@ int launch_f32x_cfg(kh::Device* d, const __bf16* pa, const __bf16* pb, int64_t M
 // workgroup takes 4 LC columns (LC lanes of one float4 each; its 256 / LC lane
 // groups take every (256 / LC)-th k) of kper rows of B, MR rows of A from LDS (k-
 // major, so a k's values are one broadcast read), eight or sixteen float4 of B in
-// flight a lane; the groups' sums meet in LDS.  Bound: the bytes of B (1 x 4096 x 4096: 341 -> 24 us, 2.8 TB/s, a third of it the sum of 32 partials; 16 rows 32, 32 rows 44, where the split product took 63).
+// flight a lane; the groups' sums meet in LDS.  Bound: the bytes of B.  1 x 4096 x
+// 4096 341 -> 24 us (2.8 TB/s, the sum of 32 partials behind it), 16 rows 342 ->
+// 32, 32 rows 344 -> 44, where the split product took 63.
 // ---------------------------------------------------------------------------
 constexpr int kRowsMost = 32, kRowsK = 512, kRowsSplits = 32;
 

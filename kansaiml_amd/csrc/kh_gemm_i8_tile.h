@@ -335,12 +335,13 @@ int launch_tile_cfg(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, 
 int64_t tiles64(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 63) / 64); }
 
 // Where the tiles below beat the ping-pong kernel's, which are at least 128 x
-// 128 and run one or two workgroups to a CU: up to six 64 x 64 tiles per CU.
+// 128 and run one or two workgroups to a CU: up to four 64 x 64 tiles per CU.
 // At K = 4096: 256 tiles (M = N = 1024) 24.7 -> 10.6 us, 512 (1024 x 2048)
-// 25.5 -> 17.4, 1024 (1024 x 4096) 30.0 -> 27.3, 1536 (4096 x 1536) 44.4 ->
-// 39.5; 2048 (2048 x 4096) 53.7 against 56.3.
+// 25.5 -> 17.4, 1024 (1024 x 4096) 30.0 -> 27.3.  Beyond it depends on how either's
+// last round fills: 1173 tiles (1472 x 3246 x 3648) 39.0 against 40.7, 1536 (4096 x
+// 1536) 44.4 against 39.5, 2048 (2048 x 4096) 53.7 against 56.3.
 bool tile_pays(const kh::Device* d, int64_t M, int64_t N, int64_t K) {
-    return tiles64(M, N) <= 6 * (int64_t)d->cus && K <= 0x7FFFFFFF / 128 && M <= 0x7FFFFFFF && N <= 0x7FFFFFFF;
+    return tiles64(M, N) <= 4 * (int64_t)d->cus && K <= 0x7FFFFFFF / 128 && M <= 0x7FFFFFFF && N <= 0x7FFFFFFF;
 }
 
 int launch_pingpong(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
@@ -365,8 +366,9 @@ int launch_pingpong(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, 
 //
 // Padded: rows that the large tiles cannot take (K no multiple of 64, or
 // unaligned) are first copied to a multiple of 64 where the product is large
-// enough to pay for the copy, more than 4 tiles per CU for unaligned rows and 6
-// for aligned ones (pooled memory, so not where the caller cannot allocate).
+// enough to pay for the copy, more than 4 tiles per CU (6 for aligned rows, which
+// the 128 x 64 tiles take as they lie); pooled memory, so not where the caller
+// cannot allocate.
 int launch_tile(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K, const Epilogue& ep,
                 bool may_alloc, unsigned* parts, int max_parts, int* nparts, bool* parts_done) {
     KH_REQUIRE(M <= 0x7FFFFFFF && N <= 0x7FFFFFFF && tiles64(M, N) <= 0x7FFFFFFF, "kh_gemm_i8: shape too large");
@@ -384,12 +386,9 @@ int launch_tile(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, int6
         rc = kh::launch_status("pad_rows");
         if (!rc) {
             const bool fused = parts && ((M + 127) / 128) * ((N + 127) / 128) <= max_parts;
-            if (tile_pays(d, M, N, Kp)) rc = launch_tile_cfg<128, 64, 2, true>(d, pa, pb, M, N, Kp, ep, 1, nullptr);
-            else {
-                rc = launch_pingpong(d, pa, pb, M, N, Kp, ep, fused ? parts : nullptr, fused ? nparts : nullptr,
-                                     kh::quant::kOutStore);
-                *parts_done = fused;
-            }
+            rc = launch_pingpong(d, pa, pb, M, N, Kp, ep, fused ? parts : nullptr, fused ? nparts : nullptr,
+                                 kh::quant::kOutStore);
+            *parts_done = fused;
         }
         kh_free(pad);  // stream-ordered: reused only by work queued after the product
         return rc;
