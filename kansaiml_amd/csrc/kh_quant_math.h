@@ -76,7 +76,7 @@ __device__ __forceinline__ Scale make_scale(unsigned mbits) {
     return r;
 }
 
-__device__ __forceinline__ void flag_nonfinite(unsigned* fault) { atomicOr(fault, kh::kFaultNonFinite); }
+__device__ __forceinline__ void flag_nonfinite(unsigned* fault) { kh::flag_fault(fault, kh::kFaultNonFinite); }
 
 // quantize.py:69 exactly: binary64 divide, rint (ties to even), clamp.
 __device__ __forceinline__ int quant_exact(float v, double s) {

@@ -106,9 +106,13 @@ int init_slot(int dev) {
     // Default priority on purpose (all streams at one priority).
     rc = hip_status(hipStreamCreateWithFlags(&s.dev.stream, hipStreamNonBlocking), "hipStreamCreate");
     if (rc) return rc;
-    rc = hip_status(hipMalloc(reinterpret_cast<void**>(&s.dev.fault), 256), "hipMalloc(fault word)");
+    rc = hip_status(hipHostMalloc(reinterpret_cast<void**>(&s.dev.fault_host), 256,
+                                  hipHostMallocMapped | hipHostMallocCoherent),
+                    "hipHostMalloc(fault record)");
     if (rc) return rc;
-    rc = hip_status(hipMemset(s.dev.fault, 0, 256), "hipMemset(fault word)");
+    std::memset(s.dev.fault_host, 0, 256);
+    rc = hip_status(hipHostGetDevicePointer(reinterpret_cast<void**>(&s.dev.fault), s.dev.fault_host, 0),
+                    "hipHostGetDevicePointer(fault record)");
     if (rc) return rc;
     // With `dev` current: this device's copy of the fixed no-alloc array.
     void* na = nullptr;
@@ -280,18 +284,13 @@ int kh_synchronize(void) {
     KH_NOT_CAPTURING(d, "kh_synchronize");
     int rc = hip_status(hipStreamSynchronize(d->stream), "hipStreamSynchronize");
     if (rc) return rc;
-    unsigned fault = 0;
-    rc = hip_status(hipMemcpy(&fault, d->fault, sizeof(unsigned), hipMemcpyDeviceToHost), "read fault word");
-    if (rc) return rc;
-    if (fault) {
-        const unsigned zero = 0;
-        rc = hip_status(hipMemcpy(d->fault, &zero, sizeof(unsigned), hipMemcpyHostToDevice), "clear fault word");
-        if (rc) return rc;
-        if (fault & kh::kFaultNonFinite)
-            return fail(KH_ERR_NONFINITE, "cannot quantize a non-finite value (NaN or inf)");
-        if (fault & kh::kFaultBadIndex)
-            return fail(KH_ERR_INVALID_ARG, "embedding: token id out of range");
-    }
+    // Read and cleared in one step each: of two threads here at once, one reports.
+    bool fault[kh::kFaultWords];
+    for (int w = 0; w < kh::kFaultWords; ++w)
+        fault[w] = __atomic_exchange_n(d->fault_host + w, 0u, __ATOMIC_RELAXED) != 0;
+    if (fault[kh::kFaultNonFinite])
+        return fail(KH_ERR_NONFINITE, "cannot quantize a non-finite value (NaN or inf)");
+    if (fault[kh::kFaultBadIndex]) return fail(KH_ERR_INVALID_ARG, "embedding: token id out of range");
     return KH_OK;
 }
 

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void embedding_kernel(const int32_t* __restric
     const int c = (int)(e % D);
     const int id = ids[r];
     if (id < 0 || id >= V) {
-        atomicOr(fault, kh::kFaultBadIndex);
+        kh::flag_fault(fault, kh::kFaultBadIndex);
         out[e] = 0.0f;
         return;
     }
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void embedding4_kernel(const int32_t* __restri
     const int id = ids[r];
     f4* o = reinterpret_cast<f4*>(out) + e;
     if (id < 0 || id >= V) {
-        atomicOr(fault, kh::kFaultBadIndex);
+        kh::flag_fault(fault, kh::kFaultBadIndex);
         *o = f4{0.f, 0.f, 0.f, 0.f};
         return;
     }
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void embedding_rows_kernel(const int32_t* __re
     for (int p = 0; p < P; ++p) {
         const int r = row0 + 2 * p + half;
         if (r >= rows) continue;
-        if (bad[p] && hl == 0) atomicOr(fault, kh::kFaultBadIndex);
+        if (bad[p] && hl == 0) kh::flag_fault(fault, kh::kFaultBadIndex);
 #pragma unroll
         for (int i = 0; i < KH; ++i)
             reinterpret_cast<f4*>(out)[(int64_t)r * D4 + hl + 32 * i] =
