@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kh_common.h"
 
@@ -115,6 +116,68 @@ __global__ __launch_bounds__(256) void quant_rows_reg_kernel(const float* __rest
         const f32x4 vv =
             __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, lt * 16, i * ROW_THREADS * 16, 0));
         __builtin_amdgcn_raw_buffer_store_b32(pack4(vv, sc), qr, lt * 4, i * ROW_THREADS * 4, 0);
+    }
+}
+
+// The same for rows of any length >= 4 at any float address and any code
+// address: 16-byte loads of x at 4-byte alignment and dword stores at byte
+// alignment (both plain global accesses).  A chunk past the row's end is pulled
+// back to its last four values, so the last two chunks may overlap and store the
+// same codes; chunks wholly past it store nothing.  16384 x 4099: 144 us with one
+// value at a time, read twice; now 60.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef unsigned u32_any __attribute__((aligned(1)));
+
+template <int WAVES_PER_ROW, int VPT>
+__global__ __launch_bounds__(256) void quant_rows_any_kernel(const float* __restrict__ x, int8_t* __restrict__ q,
+                                                             double* __restrict__ scales, int64_t rows, int cols,
+                                                             unsigned* __restrict__ fault) {
+    constexpr int ROW_THREADS = 64 * WAVES_PER_ROW;
+    constexpr int ROWS_PER_BLOCK = 256 / ROW_THREADS;
+    __shared__ unsigned red[4];
+    const int lt = threadIdx.x % ROW_THREADS;
+    const int sub = __builtin_amdgcn_readfirstlane((int)threadIdx.x / ROW_THREADS);
+    const int64_t row = (int64_t)blockIdx.x * ROWS_PER_BLOCK + sub;
+    const bool active = row < rows;
+    const float* const xr = x + (active ? row : rows - 1) * cols;
+    int8_t* const qr = q + (active ? row : rows - 1) * cols;
+    f32x4 v[VPT];
+    AbsMax am;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+        v[i] = *reinterpret_cast<const f32x4_any*>(xr + min((lt + i * ROW_THREADS) * 4, cols - 4));
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) am.add4(v[i]);
+    unsigned mb = wave_max(am.bits());
+    if (WAVES_PER_ROW > 1) {
+        const int w = threadIdx.x / 64;
+        if ((threadIdx.x & 63) == 0) red[w] = mb;
+        __syncthreads();
+        const int w0 = sub * WAVES_PER_ROW;
+        mb = red[w0];
+#pragma unroll
+        for (int i = 1; i < WAVES_PER_ROW; ++i) mb = max(mb, red[w0 + i]);
+    }
+    if (!active) return;
+    const Scale sc = make_scale(mb);
+    if (lt == 0) {
+        scales[row] = sc.s;
+        if (sc.bad) flag_nonfinite(fault);
+    }
+    unsigned redo = sc.fast ? 0u : (VPT >= 32 ? ~0u : ((1u << VPT) - 1u));
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int c = (lt + i * ROW_THREADS) * 4;
+        bool ok = true;
+        const unsigned w = pack4_fast(v[i], sc.rf, ok);
+        if (!ok) redo |= 1u << i;
+        if (c < cols) *reinterpret_cast<u32_any*>(qr + min(c, cols - 4)) = w;
+    }
+    while (redo) {
+        const int i = __builtin_ctz(redo);
+        redo &= redo - 1;
+        const int c = (lt + i * ROW_THREADS) * 4, at = min(c, cols - 4);
+        if (c < cols) *reinterpret_cast<u32_any*>(qr + at) = pack4(*reinterpret_cast<const f32x4_any*>(xr + at), sc);
     }
 }
 
@@ -481,6 +544,37 @@ __global__ __launch_bounds__(256) void dequant_vec_kernel(const int8_t* __restri
                                                step * 4096, kCacheNontemporal);
 }
 
+// The same for rows of any length >= 7 at any code and float address: the row's
+// values from its first 16-byte boundary on are stored as 16-byte runs (their
+// codes loaded as dwords at any address), the up to three before and behind them
+// one by one.  16384 x 4099: 136 us one value at a time, 106 with unaligned 16-byte
+// stores; now 60.
+template <int STEPS>
+__global__ __launch_bounds__(256) void dequant_any_kernel(const int8_t* __restrict__ q, int64_t cols,
+                                                          const double* __restrict__ scales, int per_row,
+                                                          float* __restrict__ out) {
+    const int64_t row = blockIdx.y;
+    const double s = scales[per_row ? row : 0];
+    const int8_t* const qr = q + row * cols;
+    float* const orow = out + row * cols;
+    const int head = (int)(-(reinterpret_cast<uintptr_t>(orow) >> 2) & 3);
+    const int64_t end = head + (cols - head) / 4 * 4;  // of the 16-byte runs (at least one)
+    const int64_t c0 = head + (int64_t)blockIdx.x * 1024 * STEPS + threadIdx.x * 4;
+    unsigned w[STEPS];
+#pragma unroll
+    for (int step = 0; step < STEPS; ++step)
+        w[step] = *reinterpret_cast<const u32_any*>(qr + min(c0 + step * 1024, end - 4));
+#pragma unroll
+    for (int step = 0; step < STEPS; ++step)
+        if (c0 + step * 1024 < end)
+            __builtin_nontemporal_store(deq4(w[step], s), reinterpret_cast<f32x4*>(orow + c0 + step * 1024));
+    if (blockIdx.x == 0 && threadIdx.x < 8) {
+        const int t = threadIdx.x & 3;
+        const int64_t c = threadIdx.x < 4 ? t : end + t;
+        if (threadIdx.x < 4 ? t < head : c < cols) orow[c] = deq_one(qr[c], s);
+    }
+}
+
 // Any shape / alignment.
 __global__ __launch_bounds__(256) void dequant_generic_kernel(const int8_t* __restrict__ q, int64_t n, int64_t cols,
                                                               const double* __restrict__ scales, int per_row,
@@ -629,29 +723,32 @@ int kh_quantize_rows(const float* x, int64_t rows, int64_t cols, int8_t* q, doub
     KH_DEVICE_OR_RETURN(d);
     if (cols == 0) return fill_scales_one(d, scales, rows);
     const bool vec = (cols % 4 == 0) && kh::aligned(x, 16) && kh::aligned(q, 4);
-    const unsigned per_row = (unsigned)rows;
-    const unsigned four_rows = (unsigned)((rows + 3) / 4);
-    const unsigned two_rows = (unsigned)((rows + 1) / 2);
+    const bool any = !vec && cols >= 4 && kh::aligned(x, 4);
     // The smallest row slot (threads x float4 per thread) that holds the row:
     // slots past the row's end still cost their loads' issue.
-    if (vec && cols <= 256)
-        quant_rows_reg_kernel<1, 1><<<four_rows, 256, 0, d->stream>>>(x, q, scales, rows, cols, d->fault);
-    else if (vec && cols <= 512)
-        quant_rows_reg_kernel<1, 2><<<four_rows, 256, 0, d->stream>>>(x, q, scales, rows, cols, d->fault);
-    else if (vec && cols <= 1024)
-        quant_rows_reg_kernel<1, 4><<<four_rows, 256, 0, d->stream>>>(x, q, scales, rows, cols, d->fault);
-    else if (vec && cols <= 1536)
-        quant_rows_reg_kernel<2, 3><<<two_rows, 256, 0, d->stream>>>(x, q, scales, rows, cols, d->fault);
-    else if (vec && cols <= 2048)
-        quant_rows_reg_kernel<2, 4><<<two_rows, 256, 0, d->stream>>>(x, q, scales, rows, cols, d->fault);
-    else if (vec && cols <= 4096)
-        quant_rows_reg_kernel<4, 4><<<per_row, 256, 0, d->stream>>>(x, q, scales, rows, cols, d->fault);
-    else if (vec && cols <= 16384)
-        quant_rows_reg_kernel<4, 16><<<per_row, 256, 0, d->stream>>>(x, q, scales, rows, cols, d->fault);
-    else if (vec && cols <= 32768)
-        quant_rows_reg_kernel<4, 32><<<per_row, 256, 0, d->stream>>>(x, q, scales, rows, cols, d->fault);
-    else
-        quant_rows_generic_kernel<<<per_row, 256, 0, d->stream>>>(x, q, scales, cols, d->fault);
+    auto go = [&](auto waves, auto vpt) {
+        constexpr int W = decltype(waves)::value, V = decltype(vpt)::value;
+        const unsigned blocks = (unsigned)((rows * W + 3) / 4);
+        if (vec) quant_rows_reg_kernel<W, V><<<blocks, 256, 0, d->stream>>>(x, q, scales, rows, cols, d->fault);
+        else quant_rows_any_kernel<W, V><<<blocks, 256, 0, d->stream>>>(x, q, scales, rows, (int)cols, d->fault);
+    };
+    using std::integral_constant;
+    using W1 = integral_constant<int, 1>;
+    using W2 = integral_constant<int, 2>;
+    using W4 = integral_constant<int, 4>;
+    if (!(vec || any) || cols > 32768)
+        quant_rows_generic_kernel<<<(unsigned)rows, 256, 0, d->stream>>>(x, q, scales, cols, d->fault);
+    else if (cols <= 256) go(W1(), integral_constant<int, 1>());
+    else if (cols <= 512) go(W1(), integral_constant<int, 2>());
+    else if (cols <= 1024) go(W1(), integral_constant<int, 4>());
+    else if (cols <= 1536) go(W2(), integral_constant<int, 3>());
+    else if (cols <= 2048) go(W2(), integral_constant<int, 4>());
+    else if (cols <= 4096) go(W4(), integral_constant<int, 4>());
+    else if (cols <= 6144) go(W4(), integral_constant<int, 6>());
+    else if (cols <= 8192) go(W4(), integral_constant<int, 8>());
+    else if (cols <= 12288) go(W4(), integral_constant<int, 12>());
+    else if (cols <= 16384) go(W4(), integral_constant<int, 16>());
+    else go(W4(), integral_constant<int, 32>());
     return kh::launch_status("quant_rows");
 }
 
@@ -716,20 +813,28 @@ int kh_quantize_tensor_packed(const float* w, int64_t k, int64_t n, int8_t* q_pa
 static int dequant(const int8_t* q, int64_t rows, int64_t cols, const double* scales, float* out, bool per_row) {
     KH_DEVICE_OR_RETURN(d);
     const bool vec = (cols % 4 == 0) && kh::aligned(q, 4) && kh::aligned(out, 16);
-    if (vec && rows <= 0x7FFFFFFFLL && (cols + kDeqPerBlock - 1) / kDeqPerBlock <= 0x7FFFFFFFLL) {
-        const int steps = cols > 3072 ? 4 : (int)((cols + 1023) / 1024);
+    const bool any = !vec && cols >= 7 && kh::aligned(out, 4);
+    if ((vec || any) && rows <= 0x7FFFFFFFLL && (cols + kDeqPerBlock - 1) / kDeqPerBlock <= 0x7FFFFFFFLL) {
+        // As few workgroups of up to 4 steps as the row needs, evenly filled.
+        const int64_t per = (cols + kDeqPerBlock - 1) / kDeqPerBlock;
+        const int steps = (int)((cols + 1024 * per - 1) / (1024 * per));
         const unsigned gx = (unsigned)((cols + 1024 * steps - 1) / (1024 * steps));
-        auto go = [&](const int8_t* qq, const double* ss, float* oo, unsigned nr) {
-            const dim3 g(gx, nr);
-            const int pr = per_row ? 1 : 0;
-            if (steps == 4) dequant_vec_kernel<4><<<g, 256, 0, d->stream>>>(qq, cols, ss, pr, oo);
-            else if (steps == 3) dequant_vec_kernel<3><<<g, 256, 0, d->stream>>>(qq, cols, ss, pr, oo);
-            else if (steps == 2) dequant_vec_kernel<2><<<g, 256, 0, d->stream>>>(qq, cols, ss, pr, oo);
-            else dequant_vec_kernel<1><<<g, 256, 0, d->stream>>>(qq, cols, ss, pr, oo);
-        };
         // grid.y is limited to 65535: walk the rows in slabs.
-        for (int64_t r0 = 0; r0 < rows; r0 += 65535)
-            go(q + r0 * cols, scales + (per_row ? r0 : 0), out + r0 * cols, (unsigned)min((int64_t)65535, rows - r0));
+        for (int64_t r0 = 0; r0 < rows; r0 += 65535) {
+            const dim3 g(gx, (unsigned)min((int64_t)65535, rows - r0));
+            const int8_t* const qq = q + r0 * cols;
+            const double* const ss = scales + (per_row ? r0 : 0);
+            float* const oo = out + r0 * cols;
+            auto go = [&](auto st) {
+                constexpr int S = decltype(st)::value;
+                if (vec) dequant_vec_kernel<S><<<g, 256, 0, d->stream>>>(qq, cols, ss, per_row ? 1 : 0, oo);
+                else dequant_any_kernel<S><<<g, 256, 0, d->stream>>>(qq, cols, ss, per_row ? 1 : 0, oo);
+            };
+            if (steps == 4) go(std::integral_constant<int, 4>());
+            else if (steps == 3) go(std::integral_constant<int, 3>());
+            else if (steps == 2) go(std::integral_constant<int, 2>());
+            else go(std::integral_constant<int, 1>());
+        }
     } else {
         const int64_t n = rows * cols;
         const int g = grid_for(n, 16, 16384);

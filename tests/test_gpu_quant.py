@@ -170,6 +170,31 @@ def test_quantize_weight_packed_edges(hip, k, n, shift):
     assert s1.numpy()[0] == es1
 
 
+@pytest.mark.parametrize("rows,cols,shift", [
+    (3, 3, 0), (5, 4, 1), (7, 5, 0), (9, 255, 0), (4, 257, 3), (3, 513, 0), (6, 1023, 0), (5, 1027, 0), (3, 1537, 0),
+    (3, 2050, 0), (5, 4097, 2), (9, 7, 0), (9, 9, 0), (3, 6147, 0), (3, 8200, 1), (2, 12289, 0), (2, 16381, 0), (2, 16386, 0), (2, 32767, 0), (2, 32770, 0), (1, 8192, 1)])
+def test_quantize_rows_any_length(hip, rows, cols, shift):
+    """Rows of any length at any float address, with exact ties, a zero row and
+    tiny values; codes and floats written one past an odd address; back again."""
+    H, D = hip
+    x = _outlier_matrix(rows, cols, seed=rows * 7 + cols)
+    x[0] = np.round(x[0] * 4) / np.float32(2)
+    x[-1] *= np.float32(1e-30)
+    if rows > 2:
+        x[1] = 0.0
+    xd = D.from_host(np.concatenate([np.full(shift, 9, np.float32), x.reshape(-1)])).view(shift, [rows, cols])
+    eq, es = O.ko_quantize_rows(x)
+    q, s = H.quantize_rows(xd)
+    np.testing.assert_array_equal(q.numpy(), eq)
+    np.testing.assert_array_equal(s.numpy(), es)
+    expect = (eq.astype(np.float64) * es[:, None]).astype(np.float32)
+    np.testing.assert_array_equal(bits32(H.dequantize_rows(q, s).numpy()), bits32(expect))
+    odd = D.from_host(np.concatenate([np.zeros(1, np.int8), eq.reshape(-1)])).view(1, [rows, cols])
+    np.testing.assert_array_equal(bits32(H.dequantize_rows(odd, s).numpy()), bits32(expect))
+    flat = H.dequantize_tensor(odd.reshape([rows * cols]), D.from_host(es[:1])).numpy()
+    np.testing.assert_array_equal(bits32(flat), bits32((eq.astype(np.float64) * es[0]).astype(np.float32).reshape(-1)))
+
+
 def test_misaligned_pointers_take_exact_generic_path(hip):
     """Offsets that break 16-byte alignment route to the scalar kernels."""
     H, D = hip
