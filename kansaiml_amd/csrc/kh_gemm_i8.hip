@@ -1052,7 +1052,8 @@ int launch_quant_rows(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M
 // at a time (2 rows x 512 B per wave instruction at K = 4096, the pattern of
 // a plain streaming read) and rearranged into B fragments through the wave's
 // own LDS region; otherwise each load is one B fragment (16 rows x 64 B).  Each wave takes its slice in chunks of C steps (8 where the
-// slice allows) and issues a chunk's loads, the activations (its first batch
+// slice allows; where K is no multiple of 512, one chunk of up to 24 whose weights
+// past K read zeros) and issues a chunk's loads, the activations (its first batch
 // of them) and the epilogue's operands first and then the weights, before its
 // first MFMA (scheduling barriers keep the compiler from interleaving them
 // with the MFMAs' waits), so the HBM stream and the L2-resident activations
@@ -1067,7 +1068,7 @@ int launch_quant_rows(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M
 typedef int i32x4v __attribute__((ext_vector_type(4)));
 constexpr int kSkinnyWaves = 8;
 
-template <int MT, int NT, int C, bool ONE, bool LEAN = false>
+template <int MT, int NT, int C, bool ONE, bool LEAN = false, bool TAIL = false>
 __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_i8_skinny_kernel(const int8_t* __restrict__ A,
                                                                            const int8_t* __restrict__ B, int M,
                                                                            int N, int K, int kslice, Epilogue ep) {
@@ -1077,7 +1078,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_i8_skinny_kernel(const
     // x 64 C bytes per instruction) and turned into B fragments through the
     // wave's own LDS region (C KiB: one pass of full-wave writes, then the
     // fragment reads).
-    constexpr bool TP = ONE && NT == 1 && MT <= 2 && (C == 4 || C == 8);
+    constexpr bool TP = ONE && !TAIL && NT == 1 && MT <= 2 && (C == 4 || C == 8);
     __shared__ i32x4v wt[TP ? kSkinnyWaves : 1][TP ? C : 1][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1086,13 +1087,14 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_i8_skinny_kernel(const
     // The launch guarantees kslice % (512 * C) == 0 and kslice > 0; saying so
     // lets the compiler load every kernel argument before the first weight
     // load instead of after a loop-skip branch.
-    __builtin_assume(kslice >= 64 * kSkinnyWaves * C);
+    // (TAIL: the slice ends anywhere inside the waves' 512 C.)
+    if constexpr (!TAIL) __builtin_assume(kslice >= 64 * kSkinnyWaves * C);
     // Activation loads in batches of up to 4 steps, each batch issued whole
     // before its MFMAs (all C at once measured slower at N = 11008).
     constexpr int AC = C < 4 ? C : 4;
     // Split K: workgroup (x, y) sums k in [y kslice, (y + 1) kslice) (kslice
     // = K without a split) and writes its int32 sums as partial y.
-    const int kper = kslice / kSkinnyWaves;  // a multiple of 64 * C; exactly 64 * C when ONE
+    const int kper = TAIL ? 64 * C : kslice / kSkinnyWaves;  // a multiple of 64 * C; exactly 64 * C when ONE
     const int k_begin = blockIdx.y * kslice + wave * kper;
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(A, (uint32_t)M * (uint32_t)K);
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(B, (uint32_t)N * (uint32_t)K);
@@ -1203,7 +1205,12 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_i8_skinny_kernel(const
 #pragma unroll
         for (int u = 0; u < NT; ++u)
 #pragma unroll
-            for (int c = 0; c < C; ++c) b[u][c] = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off[u], k0 + 64 * c, 0);
+            for (int c = 0; c < C; ++c) {
+                // TAIL: weights at k >= K read zeros, past the resource, whatever
+                // the activations there are.
+                const bool past = TAIL && k0 + 64 * c + kg >= K;
+                b[u][c] = __builtin_amdgcn_raw_buffer_load_b128(rb, past ? -16 : b_off[u], k0 + 64 * c, 0);
+            }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int c0 = 0; c0 < C; c0 += AC) {
@@ -1274,23 +1281,33 @@ __global__ __launch_bounds__(256) void skinny_splitk_epilogue_kernel(const int32
     epilogue_store(ep, idx / N, idx % N, N, sum);
 }
 
+// K no multiple of 512 as one chunk of up to 24 steps a wave, its weights past K
+// read as zeros (an offset past 2 GiB, so N K stays under it).
+constexpr int64_t kSkinnyTailK = 24 * 64 * kSkinnyWaves;
+
 bool skinny_fits(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K) {
-    return M >= 1 && M <= 64 && K > 0 && K % (64 * kSkinnyWaves) == 0 && kh::aligned(A, 16) &&
-           kh::aligned(B, 16) && M * K <= 0xFFFFFFFFLL && N * K <= 0xFFFFFFFFLL && N <= 0x7FFFFFFF;
+    return M >= 1 && M <= 64 && K > 0 && K % 16 == 0 && (K % (64 * kSkinnyWaves) == 0 || K <= kSkinnyTailK) &&
+           kh::aligned(A, 16) && kh::aligned(B, 16) && M * K <= 0xFFFFFFFFLL &&
+           N * K <= (K % (64 * kSkinnyWaves) == 0 ? 0xFFFFFFFFLL : 0x7FFFFFFFLL) && N <= 0x7FFFFFFF;
 }
 
 // Where the skinny kernel is faster than the 64 x 64 tiles
-// (kh_gemm_i8_tile.h): up to 16 rows everywhere; 17 to 32 except where a wide
-// weight takes several workgroups per CU, each reading its own copy of the
-// activations (M = 17, K = 8192, N = 11008: 26.2 against 20.3 us; K = 4096:
-// 13.4, 12.5; N = 4096: 7.5, 10.1); beyond, where four row tiles a wave halve
-// the workgroups in flight, only for short K and no more than one workgroup per
-// CU (M = 64, N = 4096: K = 512 4.0 against 4.4, 1536 6.4, 6.2, 4096 12.2, 9.7;
-// N = 11008: K = 512 6.9, 5.2, K = 1536 13.4, 6.9).
+// (kh_gemm_i8_tile.h).  A wide weight takes several workgroups per CU, each
+// reading its own copy of the activations, which the more rows and the longer K
+// cost the more; four row tiles a wave (M > 32) halve the workgroups in flight.
+//   M <= 16: everywhere but a wide weight's long K (us, skinny against tiles: 8 x
+//     11008 x 11008 30.4, 25.4; 8 x 11008 x 2176 9.5, 8.2; x 4096 12.0, 12.0; 8 x
+//     4096 x 5568 6.9, 12.6; 8 x 4096 x 11008 12.5, 14.1);
+//   M <= 32: a wide weight to K = 1535 (24 x 11008 x 704 5.0, 6.8; x 1536 8.4,
+//     7.7), others to 8192 or where K splits (24 x 4096 x 5568 8.5, 13.9; x 11008
+//     17.2, 14.8);
+//   beyond: up to one workgroup per CU and K = 1536 (48 x 4096 x 1536 5.9, 6.9; 64
+//     x 4096 x 4096 12.2, 9.7; 48 x 11008 x 1536 11.9, 7.5).
 bool skinny_pays(const kh::Device* d, int64_t M, int64_t N, int64_t K) {
-    if (M <= 16) return true;
-    const bool one_round = (N + 15) / 16 <= d->cus;
-    return M <= 32 ? one_round || K < 4096 : one_round && K < 1536;
+    const bool wide = (N + 15) / 16 > d->cus, tail = K % (64 * kSkinnyWaves) != 0;
+    if (M <= 16) return !(wide && M > 4 && (K >= 8192 || (tail && K >= 2048)));
+    if (M <= 32) return wide ? K < 1536 : K <= 8192 || !tail;
+    return !wide && K <= 1536;
 }
 
 // Split-K factor for a skinny launch: with one 16-column tile per workgroup a
@@ -1304,7 +1321,7 @@ constexpr int64_t kSplitMinK = 8192;
 int skinny_split(const kh::Device* d, int64_t N, int64_t K, bool may_alloc) {
     const int64_t tiles = (N + 15) / 16, steps = K / (64 * kSkinnyWaves);
     int S = 1;
-    if (!may_alloc || K < kSplitMinK) return 1;
+    if (!may_alloc || K < kSplitMinK || K % (64 * kSkinnyWaves)) return 1;
     while (S < 8 && tiles * S * 2 <= d->cus && steps % (2 * S) == 0) S *= 2;
     return S;
 }
@@ -1313,7 +1330,8 @@ int launch_skinny(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, in
                   const Epilogue& ep, bool may_alloc = true) {
     const int S = skinny_split(d, N, K, may_alloc);
     const int64_t kslice = K / S;
-    const int64_t steps = kslice / (64 * kSkinnyWaves);  // 64-k steps per wave
+    const int64_t steps = (kslice + 64 * kSkinnyWaves - 1) / (64 * kSkinnyWaves);  // 64-k steps per wave
+    const bool tail = kslice % (64 * kSkinnyWaves) != 0;
     Epilogue eps = ep;
     void* parts = nullptr;
     if (S > 1) {
@@ -1334,6 +1352,19 @@ int launch_skinny(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, in
                               decltype(leanv)::value><<<blocks, kSkinnyWaves * 64, 0, d->stream>>>(
             A, B, (int)M, (int)N, (int)K, (int)kslice, eps);
     };
+    auto go_tail = [&](auto mt, auto c) {
+        gemm_i8_skinny_kernel<decltype(mt)::value, 1, decltype(c)::value, true, false, true>
+            <<<(unsigned)((N + 15) / 16), kSkinnyWaves * 64, 0, d->stream>>>(A, B, (int)M, (int)N, (int)K, (int)K, eps);
+    };
+    auto pick_tail = [&](auto mt) {
+        if (steps <= 1) go_tail(mt, std::integral_constant<int, 1>());
+        else if (steps <= 2) go_tail(mt, std::integral_constant<int, 2>());
+        else if (steps <= 4) go_tail(mt, std::integral_constant<int, 4>());
+        else if (steps <= 8) go_tail(mt, std::integral_constant<int, 8>());
+        else if (steps <= 12) go_tail(mt, std::integral_constant<int, 12>());
+        else if (steps <= 16) go_tail(mt, std::integral_constant<int, 16>());
+        else go_tail(mt, std::integral_constant<int, 24>());
+    };
     auto pick = [&](auto mt) {
         using T = std::true_type;
         using F = std::false_type;
@@ -1353,9 +1384,10 @@ int launch_skinny(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, in
         else if (steps % 2 == 0) go(mt, N1(), std::integral_constant<int, 2>(), F(), F());
         else go(mt, N1(), std::integral_constant<int, 1>(), F(), F());
     };
-    if (M <= 16) pick(std::integral_constant<int, 1>());
-    else if (M <= 32) pick(std::integral_constant<int, 2>());
-    else pick(std::integral_constant<int, 4>());
+    auto run = [&](auto mt) { return tail ? pick_tail(mt) : pick(mt); };
+    if (M <= 16) run(std::integral_constant<int, 1>());
+    else if (M <= 32) run(std::integral_constant<int, 2>());
+    else run(std::integral_constant<int, 4>());
     int rc = kh::launch_status("gemm_i8_skinny");
     if (S > 1) {
         if (!rc) {

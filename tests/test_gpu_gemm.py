@@ -81,7 +81,8 @@ TILE_SHAPES = [
     (16, 1, 1), (3, 5, 2), (1, 15, 1),                                  # operands of less than 16 bytes
     (65, 70, 16), (300, 900, 112), (129, 64, 1040), (66, 200, 656),     # K % 16 == 0: a last stage partly past K
     (40, 64, 6144), (100, 33, 11008), (65, 130, 6160), (70, 65, 6151),  # split over 4, 8, 4 and 4 workgroups
-    (8, 300, 11008), (3, 4096, 704),                                    # few rows, K no multiple of 512
+    (8, 300, 11008), (3, 4096, 704), (1, 17, 16), (16, 33, 528), (5, 100, 1040), (17, 40, 2064),  # few rows, K no
+    (32, 64, 4112), (9, 50, 6160), (24, 16, 8176), (2, 31, 12272), (40, 70, 1520), (30, 48, 12304),  # multiple of 512
     (1700, 1700, 208), (1300, 2000, 384),                               # 128 x 64 tiles
     (2100, 2100, 65), (2600, 2600, 80), (2600, 2600, 77),               # rows padded first: tiles, ping-pong
 ]
