@@ -10,12 +10,17 @@
 //   (BM + BN) x 128 bytes.  16-byte chunk c of row r lies in slot
 //   c ^ ((r >> 1) & 7): two rows span the 64 banks, so 16 consecutive rows of
 //   one chunk (a quarter of a fragment read) fall on distinct banks.
-// * DMA: rows 16-byte aligned (K % 16 == 0).  Operands arrive by LDS-DMA, NS - 1
-//   stages ahead, one barrier a step: it publishes stage k and retires every
-//   read of stage k - 1, whose slot the step then refills.  Chunks at k >= K
-//   get an offset past the resource and read zeros.
+// * DMA: rows 16-byte aligned (K % 16 == 0).  Operands arrive by LDS-DMA, NS
+//   stages ahead.  A step waits for this wave's loads of stage k + 1 and its
+//   fragment reads of stage k, meets the other waves, refills the slot of stage
+//   k, reads the fragments of stage k + 1 and multiplies those of stage k.  The loop
+//   is unrolled over the ring: with the stage a run-time index a step spent more
+//   on addresses than on products (65 x 4096 x 4096: 13.6 us, at any depth of
+//   ring; unrolled 9.6).  Chunks at k >= K get an offset past the resource and
+//   read zeros.  Bound: LDS, which a step of a 64 x 64 tile writes 16 KB to and
+//   reads 32 KB from (384 cycles of the ~380 it takes alone on a CU).
 // * Otherwise (any K, any alignment) each thread loads its 16-byte chunks from
-//   their unaligned addresses one stage ahead and writes them to LDS.  An
+//   their unaligned addresses two stages ahead and writes them to LDS.  An
 //   address past the operand's last 16 bytes is pulled back to them; only the
 //   last stage holds such chunks and chunks past the row's end, so only there
 //   are bytes shifted into place and A's bytes at k >= K cleared (B's may then
@@ -39,8 +44,8 @@ __global__ __launch_bounds__(256, (BM + BN) * 128 * NS <= 53248 ? 3 : (BM + BN) 
     constexpr int BK = 128, kTM = BM / 64, kTN = BN / 64;
     constexpr int kLdsA = BM * BK, kStage = (BM + BN) * BK;
     constexpr int kAInst = BM / 32, kBInst = BN / 32;  // 16-byte chunks per lane and stage
-    constexpr int kLoads = kAInst + kBInst, kMost = NS - 1 > 3 ? NS - 1 : 3;
-    static_assert(DMA ? (NS >= 2 && NS <= 8) : NS == 2, "wait_loads_beyond covers up to 3 stages ahead");
+    constexpr int kLoads = kAInst + kBInst;
+    static_assert(NS == 2 || (DMA && NS == 4), "a turn of the ring below");
     __shared__ __attribute__((aligned(1024))) int8_t lds[NS * kStage];
 
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
@@ -156,7 +161,7 @@ __global__ __launch_bounds__(256, (BM + BN) * 128 * NS <= 53248 ? 3 : (BM + BN) 
 #pragma unroll
         for (int s = 0; s < NS; ++s)
             if (kt0 + s < kt1) issue(kt0 + s, s);
-        wait_loads_beyond<kLoads, kMost>(min(NS - 1, kt1 - 1 - kt0));
+        wait_loads_beyond<kLoads>(min(NS - 1, kt1 - 1 - kt0));
         meet();
         read(lds, f0);
         // Step j of a turn of the ring (kt = kt0 + j mod NS).  Steady: every
@@ -166,7 +171,7 @@ __global__ __launch_bounds__(256, (BM + BN) * 128 * NS <= 53248 ? 3 : (BM + BN) 
             if constexpr (decltype(steady)::value)
                 __builtin_amdgcn_s_waitcnt(wait_imm((NS - 2) * kLoads, 15));
             else
-                wait_loads_beyond<kLoads, kMost>(max(0, min(NS - 2, kt1 - 2 - kt)));
+                wait_loads_beyond<kLoads>(max(0, min(NS - 2, kt1 - 2 - kt)));
             meet();  // stage kt + 1 landed, stage kt read
             if (decltype(steady)::value || kt + NS < kt1) issue(kt + NS, j);
             if (decltype(steady)::value || kt + 1 < kt1) read(lds + (j + 1) % NS * kStage, next);
@@ -174,7 +179,6 @@ __global__ __launch_bounds__(256, (BM + BN) * 128 * NS <= 53248 ? 3 : (BM + BN) 
             multiply(cur);
             __builtin_amdgcn_sched_barrier(0);
         };
-        static_assert(NS == 2 || NS == 4, "a turn of the ring below");
         using std::integral_constant;
         int kt = kt0;
         for (; kt + 2 * NS <= kt1; kt += NS) {
@@ -337,11 +341,14 @@ int64_t tiles64(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 63) / 64)
 // Where the tiles below beat the ping-pong kernel's, which are at least 128 x
 // 128 and run one or two workgroups to a CU: up to four 64 x 64 tiles per CU.
 // At K = 4096: 256 tiles (M = N = 1024) 24.7 -> 10.6 us, 512 (1024 x 2048)
-// 25.5 -> 17.4, 1024 (1024 x 4096) 30.0 -> 27.3.  Beyond it depends on how either's
-// last round fills: 1173 tiles (1472 x 3246 x 3648) 39.0 against 40.7, 1536 (4096 x
-// 1536) 44.4 against 39.5, 2048 (2048 x 4096) 53.7 against 56.3.
+// 25.5 -> 17.4, 1024 (1024 x 4096) 30.0 -> 27.3.  Up to six where the 128 x 64 tiles
+// come to a full round of three workgroups to a CU (768 of them: 16384 x 384 x 1536
+// with a residual 22.3 -> 20.6, 4096 x 1536 x 4096 44.4 -> 39.5; 612: 1472 x 3246 x
+// 3648 39.0 against 40.7); 2048 tiles (2048 x 4096 x 4096) 53.7 against 56.3.
 bool tile_pays(const kh::Device* d, int64_t M, int64_t N, int64_t K) {
-    return tiles64(M, N) <= 4 * (int64_t)d->cus && K <= 0x7FFFFFFF / 128 && M <= 0x7FFFFFFF && N <= 0x7FFFFFFF;
+    if (K > 0x7FFFFFFF / 128 || M > 0x7FFFFFFF || N > 0x7FFFFFFF) return false;
+    const int64_t tiles = tiles64(M, N), wide = ((M + 127) / 128) * ((N + 63) / 64), cus = d->cus;
+    return tiles <= 4 * cus || (tiles <= 6 * cus && K > 512 && wide <= 3 * cus && 10 * wide >= 27 * cus);
 }
 
 int launch_pingpong(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
@@ -353,9 +360,11 @@ int launch_pingpong(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, 
 // Tile: 64 x 64 with four stages (two workgroups of 64 KB to a CU) up to 2.5
 // tiles per CU; beyond, 128 x 64 with two (three of 48 KB), which reads a
 // quarter less LDS per product: 1024 x 4096 x 4096 31.7 -> 27.3 us, 4096 x 1536
-// x 4096 46.5 -> 39.5, but 1024 x 2048 x 4096 17.4 against 22.4.  Unaligned rows
-// take 64 x 64 (1000 x 1250 x 1001 12.4 us, where a byte-wise gather took 165;
-// 128 x 64 14.4).
+// x 4096 46.5 -> 39.5, but 1024 x 2048 x 4096 17.4 against 22.4.  K <= 512 fills no
+// ring of four: 64 x 64 with two stages, three workgroups to a CU, up to three
+// tiles per CU (2048 x 1152 x 384 7.8 -> 6.4, 2048 x 1536 x 384 10.3 -> 8.1; 128 x 64:
+// 7.1, 9.4).  Unaligned rows take 64 x 64 (1000 x 1250 x 1001 12.4 us, where a
+// byte-wise gather took 165; 128 x 64 14.4).
 //
 // Split K: a few tiles of a long K leave CUs idle, each a chain of K / 128 steps
 // of ~0.18 us; the second launch and the partials' round trip cost ~4 us.  Split
@@ -393,7 +402,8 @@ int launch_tile(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, int6
         kh_free(pad);  // stream-ordered: reused only by work queued after the product
         return rc;
     }
-    if (dma && tiles > cus * 5 / 2) {
+    const bool brief = dma && K <= 512;
+    if (dma && tiles > (brief ? 3 * cus : cus * 5 / 2)) {
         const int64_t grid = ((M + 127) / 128) * ((N + 63) / 64);
         *parts_done = parts && grid <= max_parts;
         if (*parts_done) *nparts = (int)grid;
@@ -425,8 +435,9 @@ int launch_tile(kh::Device* d, const int8_t* A, const int8_t* B, int64_t M, int6
     *parts_done = parts && tiles <= max_parts;
     if (*parts_done) *nparts = (int)tiles;
     unsigned* const p = *parts_done ? parts : nullptr;
-    return dma ? launch_tile_cfg<64, 64, 4, true>(d, A, B, M, N, K, ep, 1, p)
-               : launch_tile_cfg<64, 64, 2, false>(d, A, B, M, N, K, ep, 1, p);
+    return brief ? launch_tile_cfg<64, 64, 2, true>(d, A, B, M, N, K, ep, 1, p)
+           : dma ? launch_tile_cfg<64, 64, 4, true>(d, A, B, M, N, K, ep, 1, p)
+                 : launch_tile_cfg<64, 64, 2, false>(d, A, B, M, N, K, ep, 1, p);
 }
 
 }  // namespace

@@ -187,7 +187,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w8_kernel(const __bf16* __restric
     constexpr int BK = 64, kTM = BM / 64, kTN = BN / 64;
     constexpr int kPlane = BM * 128, kLdsB = 3 * kPlane, kStage = kLdsB + BN * BK;
     constexpr int kAInst = BM / 32, kBInst = BN / 64;  // LDS-DMA instructions per wave: per plane, and of codes
-    constexpr int kLoads = 3 * kAInst + kBInst, kMost = NS - 1 > 3 ? NS - 1 : 3;
+    constexpr int kLoads = 3 * kAInst + kBInst;
     static_assert(NS == 2 || NS == 4, "a turn of the ring below");
     __shared__ __attribute__((aligned(1024))) int8_t lds[NS * kStage];
 
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w8_kernel(const __bf16* __restric
 #pragma unroll
     for (int s = 0; s < NS; ++s)
         if (kt0 + s < kt1) issue(kt0 + s, s);
-    wait_loads_beyond<kLoads, kMost>(min(NS - 1, kt1 - 1 - kt0));
+    wait_loads_beyond<kLoads>(min(NS - 1, kt1 - 1 - kt0));
     meet();
     read(lds, f0);
     // Step j of a turn of the ring (kt = kt0 + j mod NS).  Steady: every stage it
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w8_kernel(const __bf16* __restric
         if constexpr (decltype(steady)::value)
             __builtin_amdgcn_s_waitcnt(wait_imm((NS - 2) * kLoads, 15));
         else
-            wait_loads_beyond<kLoads, kMost>(max(0, min(NS - 2, kt1 - 2 - kt)));
+            wait_loads_beyond<kLoads>(max(0, min(NS - 2, kt1 - 2 - kt)));
         meet();  // stage kt + 1 landed, stage kt read
         if (decltype(steady)::value || kt + NS < kt1) issue(kt + NS, j);
         if (decltype(steady)::value || kt + 1 < kt1) read(lds + (j + 1) % NS * kStage, next);

@@ -37,15 +37,9 @@ __host__ __device__ constexpr int wait_imm(int vm, int lgkm) {
 }
 
 // Waits until this wave has at most `stages` x `per_stage` LDS-DMA loads in
-// flight (stages in 0..kMost, at most 3 unless said otherwise; uniform branch
-// on a wave-uniform value).
-template <int per_stage, int kMost = 3>
+// flight (stages in 0..3; uniform branch on a wave-uniform value).
+template <int per_stage>
 __device__ __forceinline__ void wait_loads_beyond(int stages) {
-    static_assert(kMost >= 3 && kMost <= 7 && kMost * per_stage <= 63, "vmcnt counts to 63");
-    if constexpr (kMost > 3) {
-        if (stages >= kMost) return __builtin_amdgcn_s_waitcnt(wait_imm(kMost * per_stage, 15));
-        if constexpr (kMost > 4) return wait_loads_beyond<per_stage, kMost - 1>(stages);
-    }
     if (stages >= 3) __builtin_amdgcn_s_waitcnt(wait_imm(3 * per_stage, 15));
     else if (stages == 2) __builtin_amdgcn_s_waitcnt(wait_imm(2 * per_stage, 15));
     else if (stages == 1) __builtin_amdgcn_s_waitcnt(wait_imm(per_stage, 15));
