@@ -320,7 +320,7 @@ def bench_skinny(steps, warmup, rows=None):
             out_rows.append({"M": M, "K": K, "N": N, "us": round(us, 2), "us_stream": round(us_stream, 2),
                              "us_single": round(us_single, 2),
                              "GB/s": round(gbs, 1), "TOPS": round(2.0 * M * N * K / (us * 1e-6) / 1e12, 2),
-                             "path": "fused decode kernel" if M <= 3 else "quantize_rows + skinny GEMM",
+                             "path": "fused decode kernel" if M <= 3 else "quantize_rows + int8 GEMM",
                              "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS,
                                           "unit": "GB/s", "frac": round(gbs / PEAK_HBM_GBS, 4),
                                           "traffic": measured_traffic(key), "traffic_key": key}})
@@ -602,13 +602,14 @@ def bench_copy(steps, warmup):
     return ms, 2.0 * COPY_BYTES / (ms * 1e-3) / 1e9
 
 
-# Kernel-name fragments (rocprofv3 Kernel_Name) of the kernels each bench line measures.
+# Kernel-name fragments (rocprofv3 Kernel_Name) of the kernels each bench line measures: the bytes of one
+# launch of each are added up.
 KERNELS = {
-    "gemm_i8_8192": "gemm_i8_pingpong_kernel",
-    "quant_rows_16384": "quant_rows_reg_kernel<4, 16>",
-    "dequant_rows_16384": "dequant_vec_kernel",
-    "fp32_matmul_4096": "gemm_f32_",
-    "copy_1GiB": "copy16_kernel",
+    "gemm_i8_8192": ("gemm_i8_pingpong_kernel",),
+    "quant_rows_16384": ("quant_rows_reg_kernel<4, 16>",),
+    "dequant_rows_16384": ("dequant_vec_kernel",),
+    "fp32_matmul_4096": ("split_units_kernel", "gemm_f32x_kernel"),
+    "copy_1GiB": ("copy16_kernel",),
 }
 ALGO_BYTES = {"gemm_i8_8192": 2 * 8192 * 8192 + 4 * 8192 * 8192, "quant_rows_16384": 5 * 16384 * 16384,
               "dequant_rows_16384": 5 * 16384 * 16384, "copy_1GiB": 2 * COPY_BYTES,
@@ -798,12 +799,12 @@ def _summarize_traffic(root, traffic):
     ff, wf = cal["fetch_factor"], cal["write_factor"]
     disp = _per_dispatch(root, ["fetch", "write"])
     rows = []
-    for key, frag in KERNELS.items():
-        f = [d["FETCH_SIZE"] for d in disp.values() if frag in d["kernel"] and "FETCH_SIZE" in d]
-        w = [d["WRITE_SIZE"] for d in disp.values() if frag in d["kernel"] and "WRITE_SIZE" in d]
-        if not f or not w or key == "copy_1GiB":
+    for key, frags in KERNELS.items():
+        f = [[d["FETCH_SIZE"] for d in disp.values() if frag in d["kernel"] and "FETCH_SIZE" in d] for frag in frags]
+        w = [[d["WRITE_SIZE"] for d in disp.values() if frag in d["kernel"] and "WRITE_SIZE" in d] for frag in frags]
+        if not all(f) or not all(w) or key == "copy_1GiB":
             continue
-        fk, wk = sum(f) / len(f), sum(w) / len(w)
+        fk, wk = (sum(sum(v) / len(v) for v in c) for c in (f, w))
         b = fk * 1024 * ff + wk * 1024 * wf
         traffic[key] = {"FETCH_SIZE_KiB": fk, "WRITE_SIZE_KiB": wk, "bytes_per_launch": b,
                         "algorithmic_bytes": ALGO_BYTES[key], "ratio": b / ALGO_BYTES[key]}
@@ -832,7 +833,7 @@ def _summarize_traffic(root, traffic):
             + _md_table(["kernel", "FETCH_SIZE KiB", "WRITE_SIZE KiB", "HBM GB/launch", "algorithmic GB", "ratio"], rows))
     cmds = [profile_command("fetch"), profile_command("write")]
     if c5:
-        body += ("\n\nC5 rows (`kh_linear_i8`, per call: the per-row quantize and the skinny GEMM for M > 2, the "
+        body += ("\n\nC5 rows (`kh_linear_i8`, per call: the per-row quantize and the int8 GEMM for M > 3, the "
                  "fused decode kernel for M <= 3; algorithmic bytes N*K + 8N + 6MK + 4MN):\n\n"
                  + _md_table(["row", "kernels", "FETCH_SIZE KiB", "WRITE_SIZE KiB", "HBM MB/call", "algorithmic MB",
                               "ratio"], c5))
